@@ -7,6 +7,7 @@ memory and streams; the computation is the gfx950 kernels of the library.
 from __future__ import annotations
 
 import ctypes
+import threading
 
 import torch
 
@@ -96,29 +97,52 @@ def gemm_column_split(m: int, n: int, k_pad: int, cus: int = 0) -> int:
 # streams get their own. Under HIP graph capture none is made or grown (the
 # zeroing would run only at replay, and eager calls would find the counters
 # dirty); a captured call runs unsplit unless the stream already has a large
-# enough workspace, which the graph then reuses on every replay.
+# enough workspace, which the graph then reuses on every replay. Graphs
+# captured on one stream therefore share its workspace: replays of them that
+# overlap (on other streams, or with eager calls on that stream) are calls
+# that overlap on one workspace.
 _workspaces: dict[tuple[int, int], torch.Tensor] = {}
+
+# Workspaces that a larger one replaced. A graph captured earlier holds the
+# address of the one its stream had then and writes there on every replay, and
+# nothing tells this module when the graph is gone, so a replaced workspace is
+# kept until the process ends. Each new one is at least twice the size of the
+# one it replaces, so a stream's kept ones are smaller than its current one.
+_retired: list[torch.Tensor] = []
+
+
+_growing = threading.Lock()
+
+
+def _stream_workspace(table: dict, device: torch.device, nbytes: int, least: int) -> torch.Tensor | None:
+    """`table`'s zeroed workspace of at least nbytes (and `least`) for the
+    current stream on `device`; None when one would have to be made or grown
+    during graph capture."""
+    dev = torch.device(device)
+    index = dev.index if dev.index is not None else torch.cuda.current_device()
+    key = (index, torch.cuda.current_stream(index).cuda_stream)
+    ws = table.get(key)
+    if ws is not None and ws.numel() >= nbytes:
+        return ws
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    with _growing:
+        ws = table.get(key)
+        if ws is not None and ws.numel() >= nbytes:
+            return ws
+        size = max(nbytes, least if ws is None else 2 * ws.numel())
+        new = torch.zeros(size, dtype=torch.uint8, device=torch.device("cuda", index))
+        if ws is not None:
+            _retired.append(ws)
+        table[key] = new
+    return new
 
 
 def workspace_for(device: torch.device, nbytes: int) -> torch.Tensor | None:
     """This module's zeroed workspace of at least nbytes for the current
     stream on `device`; None when one would have to be made or grown during
     graph capture."""
-    dev = torch.device(device)
-    index = dev.index if dev.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(index)
-    key = (index, stream.cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is not None and ws.numel() >= nbytes:
-        return ws
-    if torch.cuda.is_current_stream_capturing():
-        return None
-    new = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=torch.device("cuda", index))
-    if ws is not None:
-        # the old buffer may still be read by work queued on this stream
-        ws.record_stream(stream)
-    _workspaces[key] = new
-    return new
+    return _stream_workspace(_workspaces, device, nbytes, 1 << 20)
 
 
 def gemm_workspace_check(workspace: torch.Tensor) -> bool:
@@ -255,29 +279,19 @@ def gemv_tiled_workspace_bytes(kind: int, m: int, k: int, rows: int) -> int:
 
 
 # The tiled GEMV's K-split workspaces, one per (device, stream), each zeroed
-# when made; every completed call leaves its workspace zero. Under graph
-# capture none is made or grown (the zeroing would run only at replay): a
-# captured split call needs the stream to have one already, from an eager call
-# on it, and raises otherwise.
+# when made and kept when replaced (_retired); every completed call leaves its
+# workspace zero. Under graph capture none is made or grown (the zeroing would
+# run only at replay): a captured split call needs the stream to have one
+# already, from an eager call on it, and raises otherwise.
 _gemv_workspaces: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def gemv_workspace_for(device: torch.device, nbytes: int) -> torch.Tensor:
-    dev = torch.device(device)
-    index = dev.index if dev.index is not None else torch.cuda.current_device()
-    stream = torch.cuda.current_stream(index)
-    key = (index, stream.cuda_stream)
-    ws = _gemv_workspaces.get(key)
-    if ws is not None and ws.numel() >= nbytes:
-        return ws
-    if torch.cuda.is_current_stream_capturing():
+    ws = _stream_workspace(_gemv_workspaces, device, nbytes, 1 << 16)
+    if ws is None:
         raise LaunchError("a split tiled GEMV under graph capture needs this stream's K-split workspace: "
                           "make one eager call of the same shape on the capturing stream first")
-    new = torch.zeros(max(nbytes, 1 << 16), dtype=torch.uint8, device=torch.device("cuda", index))
-    if ws is not None:
-        ws.record_stream(stream)
-    _gemv_workspaces[key] = new
-    return new
+    return ws
 
 
 def gemv_workspace_check(workspace: torch.Tensor) -> bool:

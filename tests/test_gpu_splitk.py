@@ -279,3 +279,46 @@ def test_split_extreme_magnitudes_at_the_largest_exact_k():
     torch.cuda.synchronize()
     assert np.array_equal(c.cpu().numpy(), exp)
     assert _state_zero(work, m, n, k, 64, 32, 16)
+
+
+def test_earlier_graph_replays_after_the_workspace_grew():
+    """Two graphs captured on one stream, the second after a larger product
+    made the stream's workspace anew: the first, which holds the earlier
+    workspace's address, still gives its bits on every replay, with tensors
+    allocated and eager calls made in between."""
+    shapes = [(32, 2048, 8192), (128, 2048, 8192)]
+    need = [hip.gemm_workspace(*s) for s in shapes]
+    assert all(sp > 1 for _, sp in need) and need[1][0] > need[0][0] > 1 << 20
+    s = torch.cuda.Stream()
+    hip._workspaces.pop((torch.cuda.current_device(), s.cuda_stream), None)
+    graphs, used = [], []
+    for i, (m, n, k) in enumerate(shapes):
+        a8, w8, as_, ws = _operands(m, n, k, 60 + i)
+        want = _bits(orc.rescale(orc.gemm_i32(a8, w8, threads=8), as_, ws))
+        d = [torch.from_numpy(x).to(DEV) for x in (a8, as_, w8, ws)]
+        out = torch.empty((m, n), dtype=torch.float32, device=DEV)
+        torch.cuda.synchronize()
+        print(f"capture {m} x {n} x {k}", flush=True)
+        with torch.cuda.stream(s):
+            hip.gemm_w8a8(*d, out=out)
+            used.append(hip.workspace_for(torch.device(DEV), 0))
+        s.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            hip.gemm_w8a8(*d, out=out)
+        graphs.append((g, d, out, want))
+    assert used[0] is not used[1]
+    for rep in range(3):
+        # the sizes of both workspaces, were they free to be handed out again
+        fill = [torch.full((w.numel(),), 0xA5, dtype=torch.uint8, device=DEV) for w in used]
+        for g, d, out, want in graphs:
+            print(f"replay {rep} of {tuple(out.shape)}", flush=True)
+            out.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(_bits(out.cpu().numpy()), want), rep
+            eager = hip.gemm_w8a8(*d)
+            torch.cuda.synchronize()
+            assert np.array_equal(_bits(eager.cpu().numpy()), want), rep
+        assert all((f == 0xA5).all().item() for f in fill), rep
+        assert all(not w[:16384].any().item() and hip.gemm_workspace_check(w) for w in used), rep
