@@ -240,8 +240,11 @@ int rocknpu_hip_gemv_q8_k_tiled(uint32_t kind, const uint8_t * w, size_t w_bytes
                                 size_t workspace_bytes, void * stream);
 
 /* Bytes of the K-split workspace a tiled call of m activation rows over K = k
- * and `rows` output rows in all (the members' n summed) needs; 0 when none of
- * its launches splits. Host code only. No counterpart in the reference. */
+ * and `rows` output rows in all needs; 0 when none of its launches splits. For
+ * a group, `rows` is the members' n summed, each rounded up to a multiple of
+ * 16: a workspace for the n summed as they are serves too, with a launch per
+ * member where it does not hold every member's last tile. Host code only. No
+ * counterpart in the reference. */
 size_t rocknpu_hip_gemv_tiled_workspace_bytes(uint32_t kind, size_t m, size_t k, size_t rows);
 
 /* Waits for `stream`, then reads and clears the workspace's error word:

@@ -946,7 +946,8 @@ int rocknpu_matmul_q_q8k_group_f32_f32(rocknpu_context* ctx, size_t count, const
         if (c == 0) continue;
         void* ws = nullptr;
         size_t ws_bytes = 0, rows = 0;
-        for (size_t i = 0; i < c; ++i) rows += wn[i];
+        // whole 16-row tiles a member, so the members share one launch
+        for (size_t i = 0; i < c; ++i) rows += rk::round_up(wn[i], 16);
         if (tiled && !gemv_split_ws(ctx, kind, m, k, rows, &ws, &ws_bytes)) return kExec;
         split |= ws != nullptr;
         const int st = tiled ? rocknpu_hip_gemv_q_f32_tiled(kind, c, w, wb, wn, k, ctx->d_act.as<float>(), k, m, out,

@@ -569,9 +569,28 @@ int launch_gemv_tiled(int kind, bool fused, GemvParams& p, hipStream_t stream) {
     int64_t tiles = 0;
     for (int i = 0; i < p.count; ++i) tiles += (p.rows[i] + kTileRows - 1) / kTileRows;
     if (const int sr = gemv_tiled_ranges(kind, p.m, p.nb); sr > 1) {
-        if (!p.split_ws || p.split_ws_bytes < gemv_tiled_split_bytes(kind, p.m, p.nb, tiles) ||
-            reinterpret_cast<uintptr_t>(p.split_ws) % 256 != 0)
-            return kStatusInvalid;
+        if (!p.split_ws || reinterpret_cast<uintptr_t>(p.split_ws) % 256 != 0) return kStatusInvalid;
+        if (p.split_ws_bytes < gemv_tiled_split_bytes(kind, p.m, p.nb, tiles)) {
+            // a workspace for the members' rows summed holds any one member's
+            // tiles, but not one partly filled tile per member: then each
+            // member is a launch of its own, with the same bits
+            int64_t rows = 0;
+            for (int i = 0; i < p.count; ++i) rows += p.rows[i];
+            const int64_t summed = (rows + kTileRows - 1) / kTileRows;
+            if (p.count == 1 || p.split_ws_bytes < gemv_tiled_split_bytes(kind, p.m, p.nb, summed))
+                return kStatusInvalid;
+            for (int i = 0; i < p.count; ++i) {
+                GemvParams a = p;
+                a.count = 1;
+                a.w[0] = p.w[i];
+                a.out[0] = p.out[i];
+                a.ldo[0] = p.ldo[i];
+                a.rows[0] = p.rows[i];
+                const int st = launch_gemv_tiled(kind, fused, a, stream);
+                if (st != kStatusOk) return st;
+            }
+            return kStatusOk;
+        }
         // waves: 8, with one block index each for ranges of at most 8 blocks
         // and two for the 9-16 of two ranges; 16 with one each for the 9-16 of
         // four ranges

@@ -274,7 +274,8 @@ def gemv_tile_weights(kind: int, w: torch.Tensor, k: int, n: int, tiled: torch.T
 
 def gemv_tiled_workspace_bytes(kind: int, m: int, k: int, rows: int) -> int:
     """Bytes of the K-split workspace a tiled GEMV call of m rows over K = k
-    and `rows` output rows in all needs (0: none of its launches splits)."""
+    and `rows` output rows in all needs (0: none of its launches splits). Each
+    member's rows counted up to a multiple of 16 keep a group one launch."""
     return int(_lib.load().rocknpu_hip_gemv_tiled_workspace_bytes(kind, m, k, rows))
 
 
@@ -321,7 +322,7 @@ def gemv_q_f32_tiled(kind: int, weights, k: int, ns, x: torch.Tensor, outs=None,
     count = len(weights)
     if outs is None:
         outs = [torch.empty((m, n), dtype=torch.float32, device=x.device) for n in ns]
-    ws, ws_bytes = _gemv_ws(kind, m, k, sum(ns), x.device, workspace)
+    ws, ws_bytes = _gemv_ws(kind, m, k, sum((n + 15) // 16 * 16 for n in ns), x.device, workspace)
     w_arr = (ctypes.c_void_p * count)(*[w.data_ptr() for w in weights])
     b_arr = (ctypes.c_size_t * count)(*[w.numel() for w in weights])
     n_arr = (ctypes.c_size_t * count)(*ns)

@@ -216,6 +216,48 @@ def test_split_grouped_equals_separate_and_q8k_input():
             _check_vs_oracle(6, ws[i], k, n, x, got)
 
 
+@pytest.mark.parametrize("kind,m,k,ns", [(4, 2, 8192, (1000, 1000)), (6, 8, 5632, (1000, 1048, 17)),
+                                         (6, 1, 8192, (1, 1, 1, 1))])
+def test_split_ragged_group_on_an_exact_workspace(kind, m, k, ns):
+    """A split group whose members end inside a 16-row tile, on a workspace
+    that holds every member's tiles (one launch) and on one for the rows as
+    summed (a launch per member): both give each member's bits alone and leave
+    the workspace zero."""
+    ws = [synth.kquant(kind, n, k, index=3550 + i) for i, n in enumerate(ns)]
+    td = [hip.gemv_tile_weights(kind, _dev(w), k, n) for w, n in zip(ws, ns)]
+    x = synth.activations(m, k, index=3560 + m)
+    alone = [hip.gemv_q_f32_tiled(kind, [t], k, [n], _dev(x))[0].cpu().numpy() for t, n in zip(td, ns)]
+    whole = hip.gemv_tiled_workspace_bytes(kind, m, k, sum(-(-n // 16) * 16 for n in ns))
+    summed = hip.gemv_tiled_workspace_bytes(kind, m, k, sum(ns))
+    assert 0 < summed < whole
+    for nbytes in (whole, summed):
+        print(f"ragged split group kind={kind} m={m} workspace={nbytes}", flush=True)
+        work = torch.zeros(nbytes, dtype=torch.uint8, device=DEV)
+        got = hip.gemv_q_f32_tiled(kind, td, k, ns, _dev(x), workspace=work)
+        torch.cuda.synchronize()
+        for i, g in enumerate(got):
+            assert np.array_equal(_bits(g.cpu().numpy()), _bits(alone[i])), (nbytes, i)
+        assert not work.any().item() and hip.gemv_workspace_check(work)
+    for i, n in enumerate(ns):
+        _check_vs_oracle(kind, ws[i], k, n, x, alone[i])
+
+
+def test_capi_ragged_split_group():
+    """A grouped decode call whose members' last tiles are partly filled: its
+    342 tiles need more than the MiB that 341, the rows as summed, fit in."""
+    k, ns, m = 8192, (2728, 2728), 8
+    ws = [synth.kquant(6, n, k, index=3570 + i) for i, n in enumerate(ns)]
+    x = synth.activations(m, k, index=3572)
+    assert (hip.gemv_tiled_workspace_bytes(6, m, k, sum(ns)) <= 1 << 20
+            < hip.gemv_tiled_workspace_bytes(6, m, k, 342 * 16))
+    outs = [np.empty((m, n), np.float32) for n in ns]
+    with Context() as c:
+        assert c.matmul_q_q8k_group(ws, [6, 6], list(ns), x, outs, k) == 0
+    for w, n, o in zip(ws, ns, outs):
+        alone = hip.gemv_q_f32_tiled(6, [hip.gemv_tile_weights(6, _dev(w), k, n)], k, [n], _dev(x))[0]
+        assert np.array_equal(_bits(o), _bits(alone.cpu().numpy()))
+
+
 def test_split_workspace_left_clear_and_dirty_detected():
     """Every completed split call leaves its workspace zero; a workspace with a
     slot left set always sets the error word (the check clears it), and the

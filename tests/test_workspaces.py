@@ -57,3 +57,39 @@ def test_streams_keep_workspaces_of_their_own(on_cpu, name, get, least):
     assert b is not a and b.numel() == least
     on_cpu.stream = 7
     assert get(dev, least) is a and len(getattr(hip, name)) == 2
+
+
+def _aligned(nbytes):
+    t = torch.zeros(nbytes + 256, dtype=torch.uint8)
+    return t[-t.data_ptr() % 256:][:nbytes]
+
+
+RAGGED = [(4, 2, 8192, [8192, 1000, 1000]), (4, 2, 8192, [5000, 5000]), (6, 8, 8192, [2728, 2728]),
+          (6, 5, 5632, [1000, 1048]), (4, 3, 5632, [17, 17, 17]), (6, 1, 14336, [1, 1, 1, 1])]
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="host buffers: without a GPU no launch can read them")
+@pytest.mark.parametrize("kind,m,k,ns", RAGGED)
+def test_ragged_groups_fit_the_workspace_asked_for(monkeypatch, kind, m, k, ns):
+    """Groups whose members end inside a 16-row tile: the launch takes the
+    workspace that the module makes for it, and one of the size the query
+    gives for the members' rows summed; one byte less is refused. Without a
+    GPU an accepted call ends as a failed launch (-3), a refused one as an
+    invalid argument (-1)."""
+    made = []
+
+    def exact(device, nbytes):
+        made.append(_aligned(nbytes))
+        return made[-1]
+
+    monkeypatch.setattr(hip, "_stream", lambda: None)
+    monkeypatch.setattr(hip, "gemv_workspace_for", exact)
+    tiled = [torch.empty(hip.gemv_tiled_bytes(kind, k, n), dtype=torch.uint8) for n in ns]
+    x = torch.zeros(m, k)
+    summed = hip.gemv_tiled_workspace_bytes(kind, m, k, sum(ns))
+    assert summed > 0
+    for workspace, status in ((None, -3), (_aligned(summed), -3), (_aligned(summed - 1), -1)):
+        with pytest.raises(hip.LaunchError, match=f"status {status}$"):
+            hip.gemv_q_f32_tiled(kind, tiled, k, ns, x, workspace=workspace)
+    # what the module makes holds every tile of one launch: no falling back to one a member
+    assert made[0].numel() == hip.gemv_tiled_workspace_bytes(kind, m, k, sum(-(-n // 16) * 16 for n in ns))
