@@ -243,8 +243,10 @@ int rocknpu_hip_gemv_q8_k_tiled(uint32_t kind, const uint8_t * w, size_t w_bytes
  * and `rows` output rows in all needs; 0 when none of its launches splits. For
  * a group, `rows` is the members' n summed, each rounded up to a multiple of
  * 16: a workspace for the n summed as they are serves too, with a launch per
- * member where it does not hold every member's last tile. Host code only. No
- * counterpart in the reference. */
+ * member where it does not hold every member's last tile. No m needs more than
+ * m = 8, but the need does not grow with m throughout (a Q4_K call of 16 rows
+ * over K = 5632 does not split, one of 8 does). Host code only. No counterpart
+ * in the reference. */
 size_t rocknpu_hip_gemv_tiled_workspace_bytes(uint32_t kind, size_t m, size_t k, size_t rows);
 
 /* Waits for `stream`, then reads and clears the workspace's error word:

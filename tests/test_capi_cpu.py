@@ -178,3 +178,13 @@ def test_tiled_split_workspace_bytes_host_side():
     assert wsb(6, 4, 16640, 4096) == 0                             # 65 blocks: unsplit
     assert wsb(4, 12, 5632, 2048) == 0                             # 9-16 rows (Q4_K): unsplit
     assert wsb(5, 4, 5632, 2048) == 0 and wsb(6, 4, 5000, 2048) == 0
+
+
+def test_tiled_split_workspace_is_largest_at_eight_rows():
+    """A workspace for min(m_max, 8) rows serves every call of up to m_max."""
+    wsb = _lib.load().rocknpu_hip_gemv_tiled_workspace_bytes
+    for kind in (4, 6):
+        for nb in (16, 17, 22, 31, 32, 48, 56, 64, 65):
+            need = [wsb(kind, m, nb * 256, 4096) for m in range(1, 41)]
+            assert all(max(need[:m]) == need[min(m, 8) - 1] for m in range(1, 41)), (kind, nb)
+    assert wsb(4, 16, 5632, 4096) == 0 < wsb(4, 8, 5632, 4096)
