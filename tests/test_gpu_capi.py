@@ -208,6 +208,33 @@ def test_f16_bridge(ctx):
     np.testing.assert_allclose(out, ref, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (3, 7, 33), (5, 97, 257), (64, 256, 48), (2, 5632, 70)])
+def test_f16_bridge_bits(ctx, m, k, n):
+    """The FP16 bridge bit for bit: activations rounded to f16, then f32 sums
+    in k order. The product of two f16 values is exact in f32 (22 bits, at
+    least 2^-48), so each term rounds once, in the addition. Subnormal f16
+    values, activations beyond f16's range (Inf) and NaN weights among them."""
+    g = np.random.default_rng(100 + k)
+    w = (g.standard_normal((n, k)) * 0.1).astype(np.float16)
+    a = g.standard_normal((m, k)).astype(np.float32)
+    w[0, 0], a[0, 0] = 3e-7, 2e-6  # subnormal in f16
+    if n > 1 and m > 1:
+        a[1, k // 2] = 7e4
+        w[n - 1, k // 3] = np.nan
+        w[n // 2, k // 2] = 0.0  # Inf x 0
+    out = np.empty((m, n), np.float32)
+    assert ctx.matmul_f16(w.view(np.uint16), a, out, k, n) == STATUS_OK
+    with np.errstate(over="ignore", invalid="ignore"):
+        ah, wf = a.astype(np.float16).astype(np.float32), w.astype(np.float32)
+        ref = np.zeros((m, n), np.float32)
+        for t in range(k):
+            ref += ah[:, t, None] * wf[None, :, t]
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(out), nan)
+    assert np.array_equal(out.view(np.uint32)[~nan], ref.view(np.uint32)[~nan])
+    assert m == 1 or (np.isinf(ref).any() and nan.any())
+
+
 @pytest.mark.parametrize("mode,k", [("1", 2048), ("all", 512), ("down", 5632), ("down", 2048)])
 def test_prefill_hilo_matches_oracle(monkeypatch, mode, k):
     """ROCKNPU_PREFILL_HILO (lib.rs:2005-2083): the prompt-path W8A8 with the two-part
